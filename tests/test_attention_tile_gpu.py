@@ -90,3 +90,23 @@ def test_scale_and_strides():
     wide = _rnd(5, 40, 24, 2 * D)
     _check(40, 8, 4, 300, q=wide[:, 3:11, :D])                # strided rows and heads
     _check(40, 8, 4, 300, q=_rnd(6, 40, D, 8).transpose(1, 2))   # copied by the entry point
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("M,Hq,Hkv,L", [(36, 32, 8, 1000), (20, 16, 2, 4000), (200, 8, 2, 200), (150, 4, 1, 12000)])
+def test_weights_keep_32_bits(M, Hq, Hkv, L, dtype):
+    """The softmax weights and their sums keep 32-bit precision: the result is
+    as near the fp64 one as its own rounding to 16 bits lets it be (2-norms;
+    weights rounded to 16 bits would add a quarter).  5% is for fp32 sums and
+    ties that round the other way."""
+    from kernels.attention_fused import BlockKVCache, block_attention
+    print(f"attn weights M={M} Hq={Hq} Hkv={Hkv} L={L} {dtype}", flush=True)
+    cache = BlockKVCache(1, Hkv, L, 32, DEV, dtype)
+    k, v, q = _rnd(1, Hkv, L, D, dtype=dtype), _rnd(2, Hkv, L, D, dtype=dtype), _rnd(3, M, Hq, D, dtype=dtype)
+    cache.store(0, k, v)
+    with torch.inference_mode():
+        got = block_attention(q, cache, 0, None, valid_len=L).view(M, Hq, D).double().cpu()
+    ref = torch.from_numpy(np.asarray(oatt.attention(q.float().cpu().numpy(), k.float().cpu().numpy(),
+                                                     v.float().cpu().numpy(), None, D ** -0.5), dtype=np.float64))
+    rounding = float((ref.to(dtype).double() - ref).norm())
+    assert float((got - ref).norm()) <= 1.05 * rounding
