@@ -36,7 +36,8 @@
 // head); each keeps an online softmax (running max and sum per row) and writes
 // its unnormalised partial output; attn_combine merges the chunks in chunk
 // order.  Both orders are fixed: bit-reproducible.  More than 32 rows per KV
-// head: attn_tile.hip, its chunks merged the same way.
+// head: attn_tile.hip or, over short contexts, attn_partial without the split
+// over waves; their chunks are merged the same way.
 #include <algorithm>
 #include <type_traits>
 
@@ -340,11 +341,14 @@ SIMSD_DEV void attn_step(const AttnArgs& a, const u32x4_t (&qf)[RBW][kDSteps], c
   }
 }
 
-// Up to 32 query rows over a long context: grid (n_chunks, Hkv), 4 waves.
-// Every wave holds all RBW row blocks and a quarter of the workgroup's key
-// chunk; the four online-softmax states merge through LDS.
+// grid (n_chunks, Hkv, row groups), 4 waves (KSPLIT) or W waves.
+//   KSPLIT (up to 32 rows): every wave holds all RBW row blocks and a quarter
+//     of the workgroup's key chunk; the four online-softmax states merge
+//     through LDS.
+//   otherwise: the waves share the key chunk and own row blocks
+//     [(z*W + w)*RBW, (z*W + w + 1)*RBW) of row group z.
 // Each wave runs its 32-key steps with the next step's K/Vt loads in flight.
-template <int DT, int RBW>
+template <int DT, int RBW, bool KSPLIT>
 __global__ __launch_bounds__(256) void attn_partial_kernel(AttnArgs a) {
   constexpr int ES = DTypeInfo<DT>::kSize;
   const int lane = threadIdx.x & 63;
@@ -353,6 +357,8 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnArgs a) {
   const int g = lane >> 4, r = lane & 15;
   const int chunk_id = blockIdx.x;
   const int h = blockIdx.y;
+  const int rb0 = KSPLIT ? 0 : ((int)blockIdx.z * nw + wv) * RBW;
+  if (!KSPLIT && rb0 * 16 >= a.rows) return;   // no rows for this wave (whole wave exits)
 
   // Q^T fragments (B operand): row = rb*16 + r, dims ds*32 + 8g .. +8
   u32x4_t qf[RBW][kDSteps];
@@ -360,7 +366,7 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnArgs a) {
   bool row_ok[RBW];
 #pragma unroll
   for (int rb = 0; rb < RBW; ++rb) {
-    const int row = rb * 16 + r;
+    const int row = (rb0 + rb) * 16 + r;
     row_ok[rb] = row < a.rows;
     const int i = row_ok[rb] ? row / (int)a.M : 0;
     tok[rb] = row_ok[rb] ? row % (int)a.M : 0;
@@ -388,8 +394,8 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnArgs a) {
   const int64_t chunk_lo = (int64_t)chunk_id * a.chunk;
   if (chunk_lo >= lv) return;   // past the valid length: the merge skips this chunk
   const int64_t chunk_hi = min(lv, chunk_lo + a.chunk);
-  const int64_t c_begin = min(chunk_hi, chunk_lo + (int64_t)wv * a.wave_chunk);
-  const int64_t c_end = min(chunk_hi, c_begin + a.wave_chunk);
+  const int64_t c_begin = KSPLIT ? min(chunk_hi, chunk_lo + (int64_t)wv * a.wave_chunk) : chunk_lo;
+  const int64_t c_end = KSPLIT ? min(chunk_hi, c_begin + a.wave_chunk) : chunk_hi;
   // the next step's loads are issued before this step's arithmetic; past
   // c_end they read zeros or stale slots, whose p is 0 and V zeroed
   StepBuf<RBW> bA, bB;
@@ -408,32 +414,46 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(AttnArgs a) {
   }
 
   const int64_t base_row = ((int64_t)h * a.n_chunks + chunk_id) * a.rows_pad;
-  // merge the four waves' states in wave order: LDS o[w][row][d], ml[w][row]
-  __shared__ __attribute__((aligned(16))) float o_sh[4][RBW * 16][kHeadDim];
-  __shared__ float2 ml_sh[4][RBW * 16];
+  if constexpr (KSPLIT) {
+    // merge the four waves' states in wave order: LDS o[w][row][d], ml[w][row]
+    __shared__ __attribute__((aligned(16))) float o_sh[4][RBW * 16][kHeadDim];
+    __shared__ float2 ml_sh[4][RBW * 16];
 #pragma unroll
-  for (int rb = 0; rb < RBW; ++rb) {
-    const int row = rb * 16 + r;
+    for (int rb = 0; rb < RBW; ++rb) {
+      const int row = rb * 16 + r;
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; ++dt)
-      *reinterpret_cast<f32x4_t*>(&o_sh[wv][row][dt * 16 + 4 * g]) = acc[rb][dt];
-    if (g == 0) ml_sh[wv][row] = make_float2(m_run[rb], l_run[rb]);
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < RBW * 16 * kHeadDim; e += blockDim.x) {
-    const int row = e / kHeadDim, d = e % kHeadDim;
-    if (row >= a.rows) continue;
-    float mx = -INFINITY;
-    for (int w = 0; w < nw; ++w) mx = fmaxf(mx, ml_sh[w][row].x);
-    float o = 0.f, l = 0.f;
-    for (int w = 0; w < nw; ++w) {
-      const float2 ml = ml_sh[w][row];
-      const float wt = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - mx);
-      o += o_sh[w][row][d] * wt;
-      l += ml.y * wt;
+      for (int dt = 0; dt < kDTiles; ++dt)
+        *reinterpret_cast<f32x4_t*>(&o_sh[wv][row][dt * 16 + 4 * g]) = acc[rb][dt];
+      if (g == 0) ml_sh[wv][row] = make_float2(m_run[rb], l_run[rb]);
     }
-    a.o_part[(base_row + row) * kHeadDim + d] = o;
-    if (d == 0) a.ml_part[base_row + row] = make_float2(mx, l);
+    __syncthreads();
+    for (int e = threadIdx.x; e < RBW * 16 * kHeadDim; e += blockDim.x) {
+      const int row = e / kHeadDim, d = e % kHeadDim;
+      if (row >= a.rows) continue;
+      float mx = -INFINITY;
+      for (int w = 0; w < nw; ++w) mx = fmaxf(mx, ml_sh[w][row].x);
+      float o = 0.f, l = 0.f;
+      for (int w = 0; w < nw; ++w) {
+        const float2 ml = ml_sh[w][row];
+        const float wt = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - mx);
+        o += o_sh[w][row][d] * wt;
+        l += ml.y * wt;
+      }
+      a.o_part[(base_row + row) * kHeadDim + d] = o;
+      if (d == 0) a.ml_part[base_row + row] = make_float2(mx, l);
+    }
+  } else {
+    // lane (g, r): acc[rb][dt][j] = O^T[dim dt*16 + 4g + j][row rb*16 + r]
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb) {
+      const int row = (rb0 + rb) * 16 + r;
+      if (!row_ok[rb]) continue;
+      float* op = a.o_part + (base_row + row) * kHeadDim;
+#pragma unroll
+      for (int dt = 0; dt < kDTiles; ++dt)
+        *reinterpret_cast<f32x4_t*>(op + dt * 16 + 4 * g) = acc[rb][dt];
+      if (g == 0) a.ml_part[base_row + row] = make_float2(m_run[rb], l_run[rb]);
+    }
   }
 }
 
@@ -1408,13 +1428,24 @@ __global__ __launch_bounds__(256) void block_mask_kernel(uint8_t* __restrict__ m
   mask[(int64_t)row * smask + col] = vis ? 1 : 0;
 }
 
-// attn_tile_kernel's costs (us): a workgroup's start and end, a round of 128
-// keys with one and with two row blocks a wave, the merge launch, a partial row
-constexpr double kAttnFixedUs = 5.0, kAttnRoundUs1 = 1.5, kAttnRoundUs2 = 2.3, kAttnMergeUs = 4.0, kAttnPartUs = 2.5e-4;
+// What the forms above 32 rows per KV head cost (us), fitted to 4700 timings
+// over 680 sizes (1 to 16 KV heads, 33 to 8000 rows, up to 11000 slots): the
+// choice by them is within 0.2% (geometric mean; at most 7%) of the best form
+// and chunking timed, and 1 of 308 sizes of up to 8 row blocks is over 2%
+// slower than the direct-load form.
+// attn_tile_kernel: a call, with one and with two row blocks a wave; each
+// further workgroup on a CU; a round of 128 keys; the merge launch, a row and a
+// partial row of it.
+constexpr double kAttnStartUs1 = 5.54, kAttnStartUs2 = 7.22, kAttnNextUs = 0.713, kAttnRoundUs1 = 2.04,
+                 kAttnRoundUs2 = 2.93, kAttnMergeUs = 2.98, kAttnRowUs = 5.64e-4, kAttnPartUs = 2.85e-4;
+// attn_partial_kernel with a wave a row block, and its merge: a call, a 32-key
+// step, a partial row, a chunk of keys.
+constexpr double kAttnDirectUs = 6.37, kAttnDirectStepUs = 0.916, kAttnDirectPartUs = 2.94e-4,
+                 kAttnDirectChunkUs = 0.0641;
 
 struct AttnPlan {
   int rows, rows_pad, rb, rbw, waves, groups, n_chunks;
-  bool ksplit, head;
+  bool ksplit, head, tile;
   int split;                  // head form: workgroups per KV head
   int fsplit;                 // the same for the fused launch (qkv_rope_attention)
   int64_t chunk, wave_chunk;
@@ -1426,8 +1457,8 @@ inline int64_t up32(int64_t n) { return (n + 31) / 32 * 32; }
 
 // Up to 32 query rows per KV head (two row blocks): four waves split each
 // workgroup's key chunk, about 256 waves in all, at least one 32-key step per
-// wave.  More rows: the row blocks spread over up to 4 waves (2 blocks per wave
-// above 4 blocks) and row groups of 8 blocks, sharing 64-key or longer chunks.
+// wave.  More rows: attn_tile_kernel or, up to 8 row blocks, attn_partial_kernel
+// with a wave a row block, whichever costs less for the lengths.
 AttnPlan attn_plan(int64_t M, int64_t Hq, int64_t Hkv, int64_t L_valid) {
   AttnPlan p{};
   const int n_rep = (int)(Hq / Hkv);
@@ -1453,14 +1484,17 @@ AttnPlan attn_plan(int64_t M, int64_t Hq, int64_t Hkv, int64_t L_valid) {
     // the merge reads, and by the merge's launch.
     const int64_t rounds = (L + 127) / 128;
     double best_us = 0;
+    p.tile = true;
     for (int rbw = 1; rbw <= 2; ++rbw) {
       const int groups = (p.rb + 4 * rbw - 1) / (4 * rbw);
       const int waves = rbw == 1 ? 4 : std::max(3, ((p.rb + groups - 1) / groups + 1) / 2);
       for (int64_t nc = 1; nc <= std::min<int64_t>(rounds, kMaxChunks); nc = nc < 8 ? nc + 1 : nc + nc / 4) {
         const int64_t per = (rounds + nc - 1) / nc, n = (rounds + per - 1) / per;
         const int64_t wgs = n * Hkv * groups;
-        double us = (double)((wgs + 255) / 256) * (kAttnFixedUs + per * (rbw == 1 ? kAttnRoundUs1 : kAttnRoundUs2));
-        if (n > 1) us += kAttnMergeUs + (double)n * Hkv * p.rows_pad * kAttnPartUs;
+        const double w = (double)((wgs + 255) / 256);      // workgroups of the fullest CU
+        double us = (rbw == 1 ? kAttnStartUs1 : kAttnStartUs2) + (w - 1) * kAttnNextUs +
+                    w * per * (rbw == 1 ? kAttnRoundUs1 : kAttnRoundUs2);
+        if (n > 1) us += kAttnMergeUs + (double)Hkv * p.rows_pad * (kAttnRowUs + n * kAttnPartUs);
         if (best_us == 0 || us < best_us) {
           best_us = us;
           p.rbw = rbw;
@@ -1468,6 +1502,30 @@ AttnPlan attn_plan(int64_t M, int64_t Hq, int64_t Hkv, int64_t L_valid) {
           p.waves = waves;
           p.chunk = per * 128;
         }
+      }
+    }
+    // attn_partial_kernel with a wave a row block, up to 8 blocks in balanced
+    // groups of at most 4 waves, over about 256 workgroups of 64-key or longer
+    // chunks: short to start, so it wins where more than one round but few
+    // chunks of keys lie before it (5 tokens x 8 heads a KV head over 500 slots
+    // 8.7 us, attn_tile_kernel 10.6; 36 rows over 500 9.3 and 10.7, over 60 7.8
+    // and 7.4, over 2000 14.1 and 13.2).  Past 8 blocks its waves' own K and V
+    // loads bound it, and it lost at all but 4 sizes timed.
+    if (p.rb <= 8) {
+      const int groups = (p.rb + 3) / 4;
+      const int64_t want = (256 + Hkv - 1) / Hkv;          // chunks per head
+      int64_t chunk = (L + want - 1) / want;
+      chunk = std::max<int64_t>((chunk + 63) / 64 * 64, 64);
+      while ((L + chunk - 1) / chunk > kMaxChunks) chunk *= 2;
+      const int64_t n = (L + chunk - 1) / chunk, w = (n * Hkv * groups + 255) / 256;
+      const double us = kAttnDirectUs + kAttnDirectStepUs * w * ((std::min(chunk, L) + kKeyStep - 1) / kKeyStep) +
+                        (double)n * Hkv * p.rows_pad * kAttnDirectPartUs + n * kAttnDirectChunkUs;
+      if (us < best_us) {
+        p.tile = false;
+        p.rbw = 1;
+        p.groups = groups;
+        p.waves = (p.rb + groups - 1) / groups;
+        p.chunk = chunk;
       }
     }
     p.wave_chunk = p.chunk;
@@ -1498,7 +1556,7 @@ AttnPlan attn_plan(int64_t M, int64_t Hq, int64_t Hkv, int64_t L_valid) {
   p.cnt_bytes = up256(Hkv * 4);
   p.o_bytes = up256(Hkv * parts * p.rows_pad * kHeadDim * 4);
   p.ml_bytes = up256(Hkv * parts * p.rows_pad * 8);
-  p.bytes = (p.head ? p.split == 1 : !p.ksplit && p.n_chunks == 1) ? 0 : p.cnt_bytes + p.o_bytes + p.ml_bytes;
+  p.bytes = (p.head ? p.split == 1 : p.tile && p.n_chunks == 1) ? 0 : p.cnt_bytes + p.o_bytes + p.ml_bytes;
   return p;
 }
 
@@ -1669,15 +1727,17 @@ extern "C" int simsd_block_attention(const void* q, int64_t sq_m, int64_t sq_h, 
       return;
     }
     if (pl.ksplit) {
-      if (pl.rbw == 2) hipLaunchKernelGGL((attn_partial_kernel<DT, 2>), grid, block, 0, st, a);
-      else hipLaunchKernelGGL((attn_partial_kernel<DT, 1>), grid, block, 0, st, a);
+      if (pl.rbw == 2) hipLaunchKernelGGL((attn_partial_kernel<DT, 2, true>), grid, block, 0, st, a);
+      else hipLaunchKernelGGL((attn_partial_kernel<DT, 1, true>), grid, block, 0, st, a);
+    } else if (!pl.tile) {
+      hipLaunchKernelGGL((attn_partial_kernel<DT, 1, false>), grid, block, 0, st, a);
     } else {
       launch_attn_tile(a, pl.rbw, pl.waves, pl.groups, static_cast<char*>(out), so_m, so_h, DT, st);
       if (pl.n_chunks == 1) return;
     }
     hipLaunchKernelGGL(attn_combine_kernel<DT>, dim3((unsigned)(M * Hq)), dim3(kHeadDim), 0, st, a.o_part,
                        a.ml_part, pl.n_chunks, pl.rows_pad, M, (int)Hq, a.n_rep, static_cast<char*>(out), so_m, so_h,
-                       a.lv_dev, pl.chunk, !pl.ksplit);
+                       a.lv_dev, pl.chunk, pl.tile);
   };
   if (dtype == kBF16) partial(std::integral_constant<int, kBF16>{});
   else partial(std::integral_constant<int, kF16>{});

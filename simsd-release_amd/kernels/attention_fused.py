@@ -19,8 +19,8 @@ slots: one workgroup per KV head over a short valid length, over a longer one
 several, the last of which merges their partials; two launches past it
 (chunked partials, then their merge).  More rows take chunked partials through
 LDS (csrc/attn_tile.hip), merged by a second launch unless one chunk covers
-the keys.  The form and the chunking follow the
-host's ``valid_len`` bound, so a caller replaying graphs over a growing
+the keys, or, up to 128 rows over short contexts, 64-key chunks without LDS.
+The form and the chunking follow the host's ``valid_len`` bound, so a caller replaying graphs over a growing
 context captures one graph per bound; ``valid_len_dev`` then lowers the
 length at run time, and the kernels trim their work to it.  The cache
 (``BlockKVCache``) keeps one copy of each KV head (no per-query-head replicas)

@@ -110,3 +110,35 @@ def test_weights_keep_32_bits(M, Hq, Hkv, L, dtype):
                                                      v.float().cpu().numpy(), None, D ** -0.5), dtype=np.float64))
     rounding = float((ref.to(dtype).double() - ref).norm())
     assert float((got - ref).norm()) <= 1.05 * rounding
+
+
+def _bytes(M, Hq, Hkv, L):
+    from kernels import _native
+    return _native.lib().simsd_block_attention_workspace_bytes(M, Hq, Hkv, L)
+
+
+def _chunked(M, Hq, Hkv, n):
+    """Workspace of n chunks of keys: counters, partials, and their maxima and sums."""
+    up = lambda b: -(-b // 256) * 256
+    rows = -(-M * Hq // Hkv // 16) * 16
+    return up(Hkv * 4) + up(Hkv * n * rows * D * 4) + up(Hkv * n * rows * 8)
+
+
+# 3 to 8 row blocks over more than one round of keys and few chunks
+SHORT = [(5, 16, 2, 505), (9, 32, 8, 509), (36, 8, 8, 540), (64, 8, 8, 264), (16, 16, 2, 216), (100, 8, 8, 300), (24, 16, 8, 248)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("M,Hq,Hkv,L", SHORT)
+def test_short_contexts_take_direct_chunks(M, Hq, Hkv, L, dtype):
+    """33 to 128 rows over short contexts: 64-key chunks, a wave a row block,
+    with masks (rows that see nothing among them) and device-side lengths
+    inside a step, inside a chunk and at its end."""
+    assert _bytes(M, Hq, Hkv, L) == _chunked(M, Hq, Hkv, -(-L // 64))
+    assert _bytes(M, Hq, Hkv, 8000) < _chunked(M, Hq, Hkv, 8000 // 64)      # longer: chunks of whole rounds
+    mask = torch.rand(M, L, device=DEV, generator=torch.Generator(device=DEV).manual_seed(4)) < 0.6
+    mask[1] = False
+    _check(M, Hq, Hkv, L, dtype=dtype)
+    _check(M, Hq, Hkv, L, mask=mask, dtype=dtype)
+    for dev_len in (1, 64, 101, 128, L - 1):
+        _check(M, Hq, Hkv, L, cap=L + 64, mask=mask, dev_len=dev_len, dtype=dtype)
