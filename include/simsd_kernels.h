@@ -106,10 +106,12 @@ int64_t simsd_thin_linear_noalloc_max_scratch_bytes(void);
 int64_t simsd_thin_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype,
                                           int block_n, int split_k, int num_waves);
 
-/* The split along K of an automatic SIMSD_BLOCK_N_TILE call over `rows` weight
- * rows (gated: gate and up rows together), for callers that size the
- * partials themselves. */
-int simsd_thin_tile_split(int64_t M, int64_t rows, int64_t K, int gated);
+/* The split along K that the tile kernel takes for these sizes, for callers
+ * that size the partials themselves: `rows` weight rows (gated: gate and up
+ * rows together); partials nonzero for simsd_thin_linear_partials, whose
+ * consumer sums them, zero for calls that sum their own (an automatic
+ * SIMSD_BLOCK_N_TILE call). */
+int simsd_thin_tile_split(int64_t M, int64_t rows, int64_t K, int partials);
 
 /* The launch geometry simsd_thin_linear picks: out4 = {rows per workgroup,
  * columns per block, waves per workgroup, split_k}.  Counterpart of

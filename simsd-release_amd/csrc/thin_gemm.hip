@@ -924,7 +924,7 @@ int plan_geometry(ThinPlan& pl, int kind, int64_t M, int64_t N, int64_t K, int d
     if (kind == 2) {
       if (split_k > 1024) return set_error("thin_linear: split_k=%d exceeds 1024", split_k);
       pl.kind = 4;
-      pl.tile = thin_tile_plan(M, N, K, glu, split_k);
+      pl.tile = thin_tile_plan(M, N, K, false, split_k);
       pl.rows = pl.tile.bn;
       pl.cb = pl.tile.bm / 16;
       pl.ks = pl.tile.waves;
@@ -1425,9 +1425,9 @@ extern "C" int simsd_thin_linear_plan(int64_t M, int64_t N, int64_t K, int dtype
   return 0;
 }
 
-extern "C" int simsd_thin_tile_split(int64_t M, int64_t rows, int64_t K, int gated) {
+extern "C" int simsd_thin_tile_split(int64_t M, int64_t rows, int64_t K, int partials) {
   if (M <= 0 || rows <= 0 || K <= 0) return 1;
-  return thin_tile_plan(M, rows, K, gated != 0, 0).split;
+  return thin_tile_plan(M, rows, K, partials != 0, 0).split;
 }
 
 extern "C" int simsd_thin_linear_silu_mul(const void* x, int64_t sxm, int64_t sxk, const void* w_gate,

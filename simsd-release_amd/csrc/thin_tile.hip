@@ -23,11 +23,12 @@
 //                      LDS, but one after the other).  Reading a k step's
 //                      operands during the products of the one before, within
 //                      a wave, cost 3 to 8% on top of that and was left out.
-// Measured in a graph over > 400 MB of weights (us, against the row-block
-// kernels): 36 tokens: gate/up 4096->2x12288 43.6 (45.3), down 12288->4096
-// 20.4 (26.2), qkv 4096->6144 11.8 (18.8), o 4096->4096 8.5 (15.0); 1024
-// tokens: gate/up 192 us, 1076 TFLOP/s (1.3 ms, 160), with 4 waves 222; down in
-// 2 partials 98 (4 waves 112), qkv 58 (75).
+// Whole calls, the sum of their partials included, in a graph over 2.5 to 7 GB
+// of weights (us, against the row-block kernels): 36 tokens: gate/up
+// 4096->2x12288 42.1 (45.3), down 12288->4096 21.8 (25.6), qkv 4096->6144 14.6
+// (17.9), o 4096->4096 11.1 (12.5); 1024 tokens: gate/up 192 us, 1076 TFLOP/s
+// (1.3 ms, 160), with 4 waves 222; down in 2 partials 98 (4 waves 112), qkv 58
+// (75), both without their sum.
 #include "simsd_kernels.h"
 #include "thin_common.hpp"
 #include "thin_tile.hpp"
@@ -161,26 +162,32 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // The tiles and what one costs, for the choice below: a workgroup's fixed
 // time, its time per stage alone on its CU and as one of two on it (us), and
-// the rate at which a whole launch streams weights (bytes / us).  Fitted to
-// 2600 measurements over 12 weight shapes x 18 token counts (9 .. 2048) x
-// splits 1 .. 8; the choice by them is within 2% (geometric mean; at most 20%)
-// of the best measured tile and split.
+// the rate at which a whole launch streams weights (bytes / us).  The first
+// four are fitted to 11500 timings of whole calls (plain, gated, and partials
+// with their consumer) over 27 weight shapes x 16 token counts (9 .. 80) x
+// splits 1 .. 8, the weights from a 1.6 GB pool: the choice by them is within
+// 1% (geometric mean; at most 14%) of the best tile and split timed.  The others
+// to 900 timings of prompts (up to 2048 tokens): within 1.3%, at most 20%.
 struct Tile {
   int wm, wn, tm, tn, st;
   int per_cu;        // workgroups a CU holds (LDS)
   float launch, wg, alone, pair, rate;
 };
 constexpr Tile kTiles[] = {
-    {2, 2, 1, 2, 4, 3, 2.3f, 0.65f, 0.25f, 0.48f, 5.2e6f},
-    {2, 2, 2, 2, 4, 2, 1.8f, 1.55f, 0.28f, 0.60f, 4.6e6f},
-    {1, 4, 4, 2, 4, 1, 0.7f, 3.4f, 0.42f, 0.42f, 4.7e6f},
-    {2, 2, 4, 2, 4, 1, 0.5f, 3.3f, 0.39f, 0.39f, 3.4e6f},
+    {2, 2, 1, 2, 4, 3, 1.94f, 0.37f, 0.277f, 0.558f, 5.81e6f},
+    {2, 2, 2, 2, 4, 2, 1.12f, 1.11f, 0.325f, 0.623f, 5.5e6f},
+    {1, 4, 4, 2, 4, 1, 0.229f, 2.49f, 0.493f, 0.493f, 5.5e6f},
+    {2, 2, 4, 2, 4, 1, 0.904f, 1.69f, 0.427f, 0.427f, 4.39e6f},
     {2, 4, 4, 2, 4, 1, 0.0f, 6.0f, 0.52f, 0.52f, 3.7e6f},
     {4, 2, 4, 4, 3, 1, 0.0f, 8.4f, 0.78f, 0.78f, 3.4e6f},
     {2, 4, 4, 4, 3, 1, 0.0f, 8.8f, 0.83f, 0.83f, 3.1e6f},
 };
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 constexpr int kCus = 256;
+constexpr double kTileFloorUs = 1.48;      // a launch, beside streaming its weights
+// summing the partials of a split: a launch of its own, or (partials calls)
+// what more of them cost the launch that consumes them; us and bytes / us
+constexpr float kSumUs = 2.21f, kSumRate = 1.84e6f, kConsumeUs = 0.147f, kConsumeRate = 0.822e6f;
 
 float tile_cost(const Tile& t, int64_t wgs, int64_t stages, double weight_bytes) {
   const double s = (double)(cdiv(stages, t.st) * t.st);
@@ -188,7 +195,8 @@ float tile_cost(const Tile& t, int64_t wgs, int64_t stages, double weight_bytes)
   const double full = t.per_cu == 1 ? t.alone : t.pair * t.per_cu / 2;
   double us = t.launch + rounds * (s * full + t.wg);
   if (rest) us += s * (rest == 1 ? t.alone : t.pair) + t.wg;
-  return (float)(us > 2.2 + weight_bytes / t.rate ? us : 2.2 + weight_bytes / t.rate);
+  const double stream = kTileFloorUs + weight_bytes / t.rate;
+  return (float)(us > stream ? us : stream);
 }
 
 template <int DT, int I, bool PARTIAL, bool GLU>
@@ -224,7 +232,7 @@ void launch_cfg(const TilePlan& p, const ThinArgs& a, bool glu, bool part, hipSt
 
 }  // namespace
 
-TilePlan thin_tile_plan(int64_t M, int64_t rows, int64_t K, bool glu, int split_k) {
+TilePlan thin_tile_plan(int64_t M, int64_t rows, int64_t K, bool partials, int split_k) {
   TilePlan best{};
   float best_us = 0.f;
   const int64_t stages = cdiv(K * 2, kTileK);
@@ -237,8 +245,7 @@ TilePlan thin_tile_plan(int64_t M, int64_t rows, int64_t K, bool glu, int split_
       if (split_k > 0 ? s > 1 : s > 1 && stages < 4 * s) continue;
       const int sp = split_k > 0 ? split_k : s;
       float us = tile_cost(t, tn * tm * sp, cdiv(stages, sp), (double)rows * K * 2);
-      // what sums the partials: the launch that consumes them or, gated, one of its own
-      if (sp > 1) us += 2.7f + (float)sp * M * rows * 4 / 4.5e6f;
+      if (sp > 1) us += (partials ? kConsumeUs : kSumUs) + (float)sp * M * rows * 4 / (partials ? kConsumeRate : kSumRate);
       if (best_us == 0.f || us < best_us) {
         best_us = us;
         best.cfg = i;

@@ -16,8 +16,8 @@ struct TilePlan {
 };
 
 // The tile and, for split_k <= 0, the split along K of a call over `rows`
-// weight rows (gated: both halves).
-TilePlan thin_tile_plan(int64_t M, int64_t rows, int64_t K, bool glu, int split_k);
+// weight rows (gated: both halves); partials: the caller's next launch sums them.
+TilePlan thin_tile_plan(int64_t M, int64_t rows, int64_t K, bool partials, int split_k);
 
 // Whether the operands fit the kernel's 32-bit offsets for any of its tiles.
 bool thin_tile_fits(int64_t M, int64_t N, int64_t K, int64_t sxm, int64_t swn, int64_t sw2n, int64_t sym, int64_t srm);

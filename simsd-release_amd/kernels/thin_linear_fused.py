@@ -28,11 +28,12 @@ load stream carries no branches.
   the 4 output columns are the (up to 4) tokens -- nothing is padded.  The
   activations of a wave's K range sit in registers and serve every 4-row
   group, so the inner loop issues weight loads only.
-* M > 48, and from 17 tokens on for gated projections and weights past 20 MB,
-  and from 9 for partials (bf16/fp16): the tile kernel (``csrc/thin_tile.hip``).
-  A workgroup computes 64 or 128 weight rows x 32 to 256 tokens; both operands
-  go from memory straight into LDS several stages ahead, and
-  ``v_mfma_f32_16x16x32_bf16`` blocks reuse each LDS operand 2 to 8 times.
+* From 17 tokens on past a weight size that falls with them (``_takes_tile``:
+  20 MiB at 17, every weight of 4 MiB past 128), and from 9 for partials
+  (bf16/fp16): the tile kernel (``csrc/thin_tile.hip``).  A workgroup computes
+  64, 128 or 256 weight rows x 32 to 256 tokens; both operands go from memory
+  straight into LDS several stages ahead, and ``v_mfma_f32_16x16x32_bf16``
+  blocks reuse each LDS operand 1 to 4 times.
 * Other M > 8 (bf16/fp16): ``v_mfma_f32_16x16x32_bf16`` with 16 weight rows as the
   A operand and up to 16 tokens per block as the B operand.  The weight is
   still read as 4 rows x 256 contiguous bytes per instruction; each wave
@@ -61,10 +62,10 @@ BLOCK_N the weight rows per workgroup (4, 8, 16, 24, 32, 64, 96 or 128; other
 values round down to one of these; at least 16 above 8 tokens; 64, 96 and 128
 apply above 8 tokens in bf16/fp16 and act as 32 elsewhere; 24 applies to the
 ungated projection above 8 tokens and acts as 16 elsewhere), BLOCK_K the K elements of
-activations a wave holds at once in the GEMV (256 or 1024),
-(BLOCK_N -1: the tile kernel, which picks its tile, and with SPLIT_K 0 its
-split, by the sizes), SPLIT_K the workgroups along K, num_warps the waves per workgroup (2, 4 or 8);
-num_stages is accepted and ignored.
+activations a wave holds at once in the GEMV (256 or 1024), SPLIT_K the workgroups along K, num_warps the waves per workgroup (2, 4 or 8);
+num_stages is accepted and ignored.  BLOCK_N -1 (``TILE``) is the tile kernel,
+which picks its tile by the sizes, and with SPLIT_K 0 its split; BLOCK_K and
+num_warps mean nothing to it.
 
 Contract (reference CONTRACT, kernels/workspace/thin_linear/CONTRACT.md:26-91):
 forward only; fp32 accumulation for bf16/fp16/fp32 inputs; deterministic
@@ -160,19 +161,26 @@ TUNED: dict[tuple[int, int], tuple[int, int, int, int, int, int]] = {
 
 # Token ranges inside an entry's envelope where another geometry wins:
 # (K, N) -> (((M_lo, M_hi), 6-tuple), ...), first match taken.  Same sweep as
-# TUNED.  At 9-16 tokens the shared-activation tiles (64 weight rows per
-# workgroup, waves splitting the rows) and, for the target's merged qkv,
+# TUNED; 33-48 tokens is the verify with committed blocks folded in (one
+# block at 36 rows), swept over rows x waves x split with 48-token column
+# blocks.  Above 8 tokens these are the shared-activation tiles (64 weight rows
+# per workgroup, waves splitting the rows) and, for the target's merged qkv,
 # 24-row tiles (256 workgroups for its 6144 rows, where 32-row tiles leave 64
 # CUs idle and 16-row tiles put two workgroups on half of them: 12.38 -> 11.62
-# us at M=16); at 5-8 tokens the merged qkv with its RMSNorm prologue, where
-# 16 rows per workgroup halve the workgroups that read both column sets' rows
-# for the statistics (7.0-7.1 against 8.0-8.9 us with 8 rows; the plain
-# projection moves by at most 0.4 us either way).  Longer weights above 16
-# tokens take the tile kernel (_takes_tile).
+# us at M=16, 15.81 -> 15.30 us at M=32); at 5-8 tokens the merged qkv with
+# its RMSNorm prologue, where 16 rows per workgroup halve the workgroups that
+# read both column sets' rows for the statistics (7.0-7.1 against 8.0-8.9 us
+# with 8 rows; the plain projection moves by at most 0.4 us either way).
 TUNED_RANGES: dict[tuple[int, int], tuple[tuple[tuple[int, int], tuple[int, int, int, int, int, int]], ...]] = {
     (2048, 4096): (((5, 8), (16, 16, 256, 1, 4, 2)),),      # merged qkv      7.1 us (M=8)
-    (4096, 6144): (((9, 16), (32, 24, 256, 1, 4, 2)),),     # merged qkv     11.6 us (M=16)
-    (12288, 4096): (((9, 16), (32, 64, 256, 4, 4, 2)),),    # down_proj      22.0 us (M=16)
+    (4096, 6144): (((9, 32), (32, 24, 256, 1, 4, 2)),       # merged qkv     11.6 / 15.3 us (M=16 / 32)
+                   ((33, 48), (64, 24, 256, 2, 2, 2))),     #                17.7 / 18.3 us (M=36 / 48)
+    (4096, 4096): (((33, 48), (64, 16, 256, 1, 4, 2)),),    # o_proj         12.7 / 13.1 us (M=36 / 48)
+    (4096, 24576): (((33, 40), (64, 32, 256, 1, 2, 2)),     # gate+up (and the gated MLP) 45.3 us (M=36)
+                    ((41, 48), (64, 96, 256, 1, 8, 2))),    #                46.2 us (M=48)
+    (12288, 4096): (((9, 32), (32, 64, 256, 4, 4, 2)),      # down_proj   22.0 / 23.3 us (M=16 / 32)
+                    ((33, 48), (64, 32, 256, 4, 2, 2))),    #             26.2 / 27.9 us (M=36 / 48)
+    (4096, 151936): (((17, 32), (32, 64, 256, 1, 4, 2)),),  # lm_head      234 us (M=32)
 }
 
 
@@ -239,25 +247,44 @@ def _rows_for(block_n: int) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
-def _tile_split(M: int, rows: int, K: int, gated: bool) -> int:
+def _tile_split(M: int, rows: int, K: int, partials: bool = False) -> int:
     """The split along K the tile kernel takes for these sizes (a pure function of them)."""
-    return _native.lib().simsd_thin_tile_split(M, rows, K, int(gated))
+    return _native.lib().simsd_thin_tile_split(M, rows, K, int(partials))
 
 
-# Where calls that reduce their own split take the tile kernel: prompts, and
-# below them weights past this many bytes from 17 tokens on.  A tile call
-# splits K over workgroups where the row-block kernels split it over waves,
-# and pays a reduce launch (~3 us) for it.  Tile against row-block, us: at 16
-# tokens 2048 -> 4096 8.1 / 5.7, 4096 -> 4096 10.7 / 8.8, 4096 -> 24576
-# 36.0 / 34.9; at 24, 2048 -> 4096 8.4 / 7.3, 6144 -> 2048 11.0 / 13.1,
-# 4096 -> 4096 10.9 / 11.0, 2048 -> 12288 12.8 / 14.8; at 36 and 48 tokens
-# 2048 -> 2048 8.8 / 8.2 and 9.4 / 8.3, 4096 -> 24576 38.2 / 43.5 and
-# 39.5 / 44.4; a 151936-row head 208 / 228 at 24, 227 / 332 at 48.
-TILE_MIN_WEIGHT_BYTES = 20 << 20
+# Where calls that reduce their own split take the tile kernel:
+# (most tokens, MiB of weight from which plain calls do, the same for gated).
+# A tile call splits K over workgroups where the row-block kernels split it
+# over waves, and pays a reduce launch (~3 us) for it, so small weights and few
+# tokens stay with those, whose cost steps with their column blocks (16, 32, 48
+# tokens, 32 past that).  Row-block over tile time at each side of the lines,
+# weights from a 1 to 7 GB pool:
+#   17-32 tokens  17 MB plain 0.92-0.94, 21 MB 1.03-1.07; gated 13 MB 0.94-1.0, 17 MB 1.12-1.19
+#   33-48         17 MB plain 0.97-1.02, 21 MB 1.09-1.14; gated 6 MB 1.08-1.17
+#   49-64         8 MB plain 0.83-1.07, 13 MB 1.07; gated 17 MB 0.96-0.99, 21 MB 1.06-1.10
+#   65-128        6 MB 0.90-1.06, 8 MB 1.02-1.17
+#   past that     2 MB over 1024 rows 0.67-0.93 (to 384 tokens), over 2048 1.1-1.8, 4 MB 1.04-1.3
+_TILE_MIN_MIB = ((32, 20, 16), (48, 20, 6), (64, 12, 20), (128, 8, 8))
+# Swept shapes whose row-block geometry keeps up all the same, (K, N): tokens.
+# At 32 tokens, row-block / tile: gate/up 38.8 / 38.9 us or, where memory runs
+# slower, 40.8 / 42.6; qkv 15.3 / 15.3 or 16.1 / 16.7.
+_ROW_BLOCK_RANGES = {(4096, 24576): (17, 32), (4096, 6144): (21, 32)}
 
 
 def _takes_tile(M: int, N_rows: int, K: int, gated: bool) -> bool:
-    return M > 48 or (M > 16 and (gated or N_rows * K * 2 >= TILE_MIN_WEIGHT_BYTES))
+    """Whether a 16-bit call on K-contiguous aligned rows takes the tile kernel."""
+    if M <= 16:
+        return False
+    lo, hi = _ROW_BLOCK_RANGES.get((K, N_rows), (0, -1))
+    # gated, up to 32 tokens: the row-block kernel streams many rows of at most
+    # 8 KB as fast (4096 -> 2 x 16000 45.2 / 49.1 us at 17 tokens, 48.9 / 50.2 at 32)
+    if lo <= M <= hi or (gated and M <= 32 and N_rows >= 24576 and K <= 4096):
+        return False
+    mib = N_rows * K * 2 / 2 ** 20
+    for most, plain, glu in _TILE_MIN_MIB:
+        if M <= most:
+            return mib >= (glu if gated else plain)
+    return mib >= 4 or N_rows >= 2048 or M > 384
 
 
 def _launch_config(M: int, N_rows: int, K: int, itemsize: int, config, num_warps, vec=None, gated: bool = False):
@@ -265,11 +292,10 @@ def _launch_config(M: int, N_rows: int, K: int, itemsize: int, config, num_warps
     bits on K-contiguous aligned rows (``vec()``; None: known to be) the tile
     kernel where it wins; else TUNED for (K, N_rows), else the heuristic."""
     if config is not None and int(config[1]) == TILE:
-        split = int(config[3]) or _tile_split(M, N_rows, K, gated)
-        return TILE, 0, split, _DEFAULT_WAVES
-    if (config is None and num_warps is None and itemsize == 2 and M > 16 and _takes_tile(M, N_rows, K, gated)
+        return TILE, 0, int(config[3]) or _tile_split(M, N_rows, K), _DEFAULT_WAVES
+    if (config is None and num_warps is None and itemsize == 2 and _takes_tile(M, N_rows, K, gated)
             and (vec is None or vec())):
-        return TILE, 0, _tile_split(M, N_rows, K, gated), _DEFAULT_WAVES
+        return TILE, 0, _tile_split(M, N_rows, K), _DEFAULT_WAVES
     if config is not None:
         block_n, block_k, split_k = int(config[1]), int(config[2]), int(config[3])
         waves = num_warps or _DEFAULT_WAVES
@@ -480,26 +506,31 @@ def thin_linear_residual(x: torch.Tensor, w: torch.Tensor, residual: torch.Tenso
 REDUCE_MAX_SPLIT = 8   # partials the consuming launches sum
 
 # Geometries of thin_linear_partials where they differ from the other calls':
-# (K, N), or None for every other shape, -> (((M_lo, M_hi), 6-tuple), ...);
-# BLOCK_N TILE: the tile kernel, its split by the sizes.  The partials pay no
-# reduce launch of their own, so a split along K costs only the consumer's
-# extra reads and the tile kernel wins from 9 tokens on (9 / 16 / 32 / 48
-# tokens against the row-block kernels' best split, us: 12288 -> 4096
-# 19.4 / 18.5 / 19.2 / 20.8 against 19.5 / 19.1 / 20.1 / 25.5, 6144 -> 2048
-# 6.5 / 6.6 / 7.0 / 7.6 against 11.4 / 12.0 / 13.4 / 17.8, 4096 -> 4096
-# 8.2 / 7.6 / 8.0 / 8.9 against 8.1 / 8.0 / 8.9 / 12.3, 2048 -> 2048
-# 3.9 / 4.1 / 4.3 / 4.8 against 4.9 / 5.0 / 6.4 / 8.2), but for the target's
-# merged qkv up to 16, whose 6144 rows are 256 tiles of 24 (10.7-11.2 against
-# 12.3-13.5).
+# (K, N), or None for every other shape of at least PARTIALS_TILE_MIN_ROWS
+# rows, -> (((M_lo, M_hi), 6-tuple), ...); BLOCK_N TILE: the tile kernel, its
+# split by the sizes.  The partials pay no reduce launch of their own, so a
+# split along K costs only the consumer's extra reads and the tile kernel wins
+# from 9 tokens on (with the consumer, 9 / 16 / 32 / 48 tokens against the
+# row-block kernels' best split, us: 12288 -> 4096 22.0 / 22.4 / 22.5 / 23.8
+# against 22.2 / 22.9 / 23.3 / 28.5, 6144 -> 2048 10.4 / 10.4 / 11.1 / 11.7
+# against 14.6 / 14.3 / 15.3 / 19.9).  Not over 1024 rows, whose 16 tiles leave
+# the chip idle at any split (4096 -> 1024 at 32 tokens 8.6 against 7.5), and
+# not up to 16 tokens over the target's merged qkv, whose 6144 rows are 256
+# tiles of 24 (10% ahead), its o (4%), or the draft's qkv and o (4%).
+PARTIALS_TILE_MIN_ROWS = 2048
 PARTIALS_RANGES: dict[tuple[int, int] | None, tuple[tuple[tuple[int, int], tuple[int, int, int, int, int, int]], ...]] = {
     (4096, 6144): (((9, 16), (64, 24, 256, 2, 2, 2)),),
+    (4096, 4096): (((9, 16), (64, 16, 256, 2, 2, 2)),),
+    (2048, 4096): (((9, 16), (16, 8, 256, 1, 4, 2)),),
+    (2048, 2048): (((9, 16), (16, 8, 1024, 1, 2, 2)),),
     None: (((9, 48), (64, TILE, 0, 0, 4, 2)),),
 }
 
 
 def _partials_config(M: int, N: int, K: int):
     """The PARTIALS_RANGES 6-tuple for this call, or None (then as the other calls)."""
-    for (lo, hi), cfg in PARTIALS_RANGES.get((K, N), ()) + PARTIALS_RANGES.get(None, ()):
+    every = PARTIALS_RANGES.get(None, ()) if N >= PARTIALS_TILE_MIN_ROWS else ()
+    for (lo, hi), cfg in PARTIALS_RANGES.get((K, N), ()) + every:
         if lo <= M <= hi:
             return cfg
     return None
@@ -527,8 +558,10 @@ def thin_linear_partials(x: torch.Tensor, w: torch.Tensor, config=None, num_warp
     dev = _native.require_device(x, w)
     if config is None and x.element_size() == 2:
         cfg = _partials_config(M, N, K)
-        if cfg is not None and (cfg[1] != TILE or (num_warps is None and _vec_rows(x) and _vec_rows(w))):
+        if cfg is not None and cfg[1] != TILE:
             config, num_warps = cfg[:4], num_warps or cfg[4]
+        elif cfg is not None and num_warps is None and _vec_rows(x) and _vec_rows(w):
+            config = (*cfg[:3], _tile_split(M, N, K, True))
     block_n, block_k, split_k, waves = _launch_config(M, N, K, x.element_size(), config, num_warps,
                                                       lambda: _vec_rows(x) and _vec_rows(w))
     split_k = max(1, min(split_k, REDUCE_MAX_SPLIT))

@@ -112,3 +112,42 @@ def test_tile_split_is_sane():
             assert s in (1, 2, 4, 8) and (s == 1 or K * 2 >= 4 * s * 128), (M, rows, K, s)
     assert lib.simsd_thin_tile_split(1024, 24576, 4096, 1) == 1
     assert lib.simsd_thin_tile_split(36, 4096, 12288, 0) > 1
+
+
+# (tokens, rows, K, gated): whether the call takes the tile kernel.  Either side
+# of each line, where the other kernel is slower.
+LINES = [((16, 24576, 4096, False), False), ((17, 4096, 2048, False), False), ((17, 4096, 2560, False), True),
+         ((32, 4096, 4096, False), True), ((32, 24576, 4096, False), False), ((36, 24576, 4096, False), True),
+         ((32, 6144, 4096, False), False), ((17, 6144, 4096, False), True), ((36, 6144, 4096, False), True),
+         ((32, 4096, 12288, False), True), ((32, 151936, 4096, False), True), ((28, 24576, 4096, True), False),
+         ((28, 12288, 2048, True), True), ((24, 6144, 1024, True), False), ((40, 3072, 1024, True), True),
+         ((49, 2048, 2048, False), False), ((64, 2048, 2048, False), False), ((65, 2048, 2048, False), True),
+         ((64, 4096, 2048, True), False), ((64, 4096, 2048, False), True), ((80, 1024, 2048, False), False),
+         ((133, 1024, 2048, False), True), ((256, 1024, 1024, False), False), ((512, 1024, 1024, False), True)]
+
+
+def test_lines_between_tile_and_row_blocks():
+    """The rule takes the kernel that was the faster on both sides of its
+    lines; partials' own rule leaves 1024-row projections and the swept shapes
+    below 17 tokens with the row blocks."""
+    from kernels.thin_linear_fused import TILE, _launch_config, _partials_config
+    for (M, rows, K, gated), tile in LINES:
+        got = _launch_config(M, rows, K, 2, None, None, gated=gated)
+        assert (got[0] == TILE) == tile, (M, rows, K, gated, got)
+        assert _launch_config(M, rows, K, 2, None, None, vec=lambda: False, gated=gated)[0] != TILE
+        assert _launch_config(M, rows, K, 4, None, None, gated=gated)[0] != TILE
+    for M, rows, K, tile in [(9, 4096, 12288, True), (48, 4096, 4096, True), (16, 6144, 4096, False), (17, 6144, 4096, True),
+                             (16, 2048, 2048, False), (17, 2048, 2048, True), (9, 4096, 2048, False), (32, 1024, 4096, False)]:
+        cfg = _partials_config(M, rows, K)
+        assert (cfg is not None and cfg[1] == TILE) == tile, (M, rows, K, cfg)
+
+
+def test_split_follows_who_sums_the_partials():
+    """A wide, deep verify projection splits K although the call sums its own
+    partials; one whose tiles fill the chip does not; a short one splits only
+    where its consumer sums them, without a launch for it."""
+    from kernels import _native
+    split = _native.lib().simsd_thin_tile_split
+    assert split(17, 6144, 4096, 0) == 4 and split(32, 8192, 2560, 0) == 2
+    assert split(28, 24576, 4096, 0) == 1 and split(36, 24576, 4096, 0) == 1
+    assert split(17, 6144, 1024, 0) == 1 and split(17, 6144, 1024, 1) == 2
