@@ -292,7 +292,10 @@ def _launch_config(M: int, N_rows: int, K: int, itemsize: int, config, num_warps
     bits on K-contiguous aligned rows (``vec()``; None: known to be) the tile
     kernel where it wins; else TUNED for (K, N_rows), else the heuristic."""
     if config is not None and int(config[1]) == TILE:
-        return TILE, 0, int(config[3]) or _tile_split(M, N_rows, K), _DEFAULT_WAVES
+        split = int(config[3])
+        if split < 0:
+            raise ValueError(f"SPLIT_K must be >= 1, or 0 with BLOCK_N {TILE}, got {split}")
+        return TILE, 0, split or _tile_split(M, N_rows, K), _DEFAULT_WAVES
     if (config is None and num_warps is None and itemsize == 2 and _takes_tile(M, N_rows, K, gated)
             and (vec is None or vec())):
         return TILE, 0, _tile_split(M, N_rows, K), _DEFAULT_WAVES

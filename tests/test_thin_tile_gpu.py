@@ -151,3 +151,12 @@ def test_split_follows_who_sums_the_partials():
     assert split(17, 6144, 4096, 0) == 4 and split(32, 8192, 2560, 0) == 2
     assert split(28, 24576, 4096, 0) == 1 and split(36, 24576, 4096, 0) == 1
     assert split(17, 6144, 1024, 0) == 1 and split(17, 6144, 1024, 1) == 2
+
+
+def test_negative_split_is_refused():
+    """A negative SPLIT_K raises before any launch, with BLOCK_N TILE as without."""
+    from kernels.thin_linear_fused import TILE, _launch_config
+    for block_n in (TILE, 16):
+        with pytest.raises(ValueError, match="SPLIT_K"):
+            _launch_config(36, 4096, 4096, 2, (64, block_n, 0, -2), None)
+    assert _launch_config(36, 4096, 4096, 2, (64, TILE, 0, 0), None)[2] == 4
