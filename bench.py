@@ -409,8 +409,8 @@ def run_layer(args, torch, dev):
         H, QKV, I, L = 4096, 6144, 12288, 36
     # four launches, plus a norm launch for each of the two norms above 8
     # rows and a reduce launch for each split-K projection
-    launches = 4 + (2 if M > 8 else 0) + sum(pick_config(M, N, K)[3] > 1
-                                             for N, K in ((QKV, H), (H, H), (2 * I, H), (H, I)))
+    launches = 4 + (2 if M > 8 else 0) + sum(pick_config(M, N, K, gated=glu)[3] > 1
+                                             for N, K, glu in ((QKV, H, False), (H, H, False), (2 * I, H, True), (H, I, False)))
     eps = 1e-6
     layers = []
     for layer in range(L):

@@ -184,12 +184,16 @@ TUNED_RANGES: dict[tuple[int, int], tuple[tuple[tuple[int, int], tuple[int, int,
 }
 
 
-def pick_config(M: int, N: int, K: int, itemsize: int = 2) -> tuple[int, int, int, int]:
-    """(BLOCK_M, BLOCK_N, BLOCK_K, SPLIT_K) -- tuned where known, else heuristic."""
+def pick_config(M: int, N: int, K: int, itemsize: int = 2, gated: bool = False) -> tuple[int, int, int, int]:
+    """(BLOCK_M, BLOCK_N, BLOCK_K, SPLIT_K) of a call on K-contiguous aligned
+    operands (gated: N gate and up rows together): the tile kernel where it is
+    taken (BLOCK_N TILE; its tile is ``simsd_thin_linear_plan``'s), else tuned
+    where known, else heuristic."""
     full = _tuned_for(M, N, K)
-    if full is not None:
-        return full[0], full[1], full[2], full[3]
-    return _heuristic_config(M, N, K, itemsize)
+    cfg = full[:4] if full is not None else _heuristic_config(M, N, K, itemsize)
+    if itemsize == 2 and _takes_tile(M, N, K, gated):
+        return cfg[0], TILE, 0, _tile_split(M, N, K)
+    return cfg
 
 
 def _tuned_for(M: int, N: int, K: int):

@@ -160,3 +160,16 @@ def test_negative_split_is_refused():
         with pytest.raises(ValueError, match="SPLIT_K"):
             _launch_config(36, 4096, 4096, 2, (64, block_n, 0, -2), None)
     assert _launch_config(36, 4096, 4096, 2, (64, TILE, 0, 0), None)[2] == 4
+
+
+@pytest.mark.parametrize("M", [4, 16, 17, 32, 36, 48, 64, 133, 1024])
+def test_pick_config_is_what_runs(M):
+    """pick_config's geometry and split are those the calls take, and passing
+    it back as the config gives the same call."""
+    from kernels.thin_linear_fused import TILE, _launch_config, pick_config
+    for K, rows in ((4096, 6144), (4096, 4096), (4096, 24576), (12288, 4096), (2048, 2048), (3000, 5000)):
+        for gated in (False, True):
+            cfg, runs = pick_config(M, rows, K, gated=gated), _launch_config(M, rows, K, 2, None, None, gated=gated)
+            assert (cfg[1] == TILE) == (runs[0] == TILE) and cfg[3] == runs[2], (M, rows, K, gated)
+            assert _launch_config(M, rows, K, 2, cfg, runs[3], gated=gated) == runs, (M, rows, K, gated)
+        assert pick_config(M, rows, K, 4)[1] != TILE
