@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define SIMSD_ABI_VERSION 18
+#define SIMSD_ABI_VERSION 19
 
 /* dtype codes */
 #define SIMSD_DTYPE_BF16 0

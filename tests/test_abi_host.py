@@ -11,6 +11,7 @@
 from __future__ import annotations
 
 import ctypes
+import hashlib
 import os
 import re
 
@@ -43,6 +44,18 @@ def test_abi_version_matches_header():
     from kernels import _native
     m = re.search(r"#define SIMSD_ABI_VERSION (\d+)", open(HEADER).read())
     assert int(m.group(1)) == _native.lib().simsd_abi_version() == _native.ABI_VERSION
+
+
+# the entry points each ABI version declares (SHA-1 of their sorted names)
+ENTRY_POINTS = {18: "f2fd83548ea2", 19: "a4ae338857a2"}
+
+
+def test_entry_points_belong_to_the_version():
+    """A library of one version has all of that version's entry points, so a
+    caller that checks the version finds every symbol it binds."""
+    from kernels import _native
+    got = hashlib.sha1(" ".join(header_functions()).encode()).hexdigest()[:12]
+    assert ENTRY_POINTS[_native.ABI_VERSION] == got, "entry points added or removed: a new SIMSD_ABI_VERSION"
 
 
 def test_header_constants_match_binding():
