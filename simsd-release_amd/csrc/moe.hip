@@ -836,16 +836,22 @@ __global__ __launch_bounds__(64 * W) void moe_down_combine_kernel(SIMSD_MOE_HOT)
   }
 }
 
-// Slots an expert holds on average from which the grouped projections take
-// runs of tiles (moe_tile.hip); below, each tile streams its expert's weights
-// by itself.  Us a layer, runs against single tiles, both with the parallel
-// scatter: 256 experts 9.4 slots 320 / 343; 128 experts 8 slots 138 / 127.
-// Runs against single tiles with the one-wave scatter (7 ns a slot more): 256
-// experts 16 slots 412 / 515, 31 slots 447 / 899; 128 experts 12.5 slots 150 /
-// 178; 64 experts 12 slots 190 / 189, 19 slots 198 / 273.
-constexpr int64_t kRunMinSlots = 10;
 // ------------------------------------------------------------------ host side
 namespace {
+
+// Slots an expert holds on average from which the grouped projections take
+// runs of tiles (moe_tile.hip); below, each tile streams its expert's weights
+// by itself, over as many more workgroups.  Experts whose columns fill the chip
+// several times (10 workgroups a CU of gate/up, one run an expert) gain from 11
+// slots on, others from 18.  Single tiles over runs, us a layer, at 10 / 11 /
+// 14 / 18 slots: 256 experts x 512 columns 1.02 1.08 1.22 1.47; 128 x 768 0.99
+// 0.98 1.12 1.43; 8 x 14336 0.96 1.03 1.11 1.47; 16 x 6400 0.98 1.00 1.19 1.33;
+// 64 x 1024 0.88 0.90 0.98 1.21; 16 x 1024 0.85 0.87 0.90 1.11; 8 x 2048 0.77
+// 0.77 0.83 1.07; 8 x 5632 0.92 0.95 1.09 1.21.
+constexpr int64_t kRunMinSlots = 11, kRunMinSlotsFew = 18, kRunColumns = 10 * 256 * 32;
+bool takes_runs(const MoeArgs& a) {
+  return a.T * a.k >= (a.E * a.I >= kRunColumns ? kRunMinSlots : kRunMinSlotsFew) * a.E;
+}
 
 inline int esize_of(int dtype) { return dtype == kF32 ? 4 : 2; }
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1111,7 +1117,7 @@ extern "C" int simsd_moe_grouped_ffn(
                      Imax * es <= 8 * kStep4Bytes && (sde * es) % 16 == 0 && (sdh * es) % 16 == 0 &&
                      (!has_shared || (shd_h * es) % 16 == 0) &&
                      units <= kSmallW * (Imax * es <= 4 * kStep4Bytes ? kSmallUM : kSmallUM8);
-  const bool tile = T * k >= kRunMinSlots * E && moe_tile_fits(a, dtype);
+  const bool tile = takes_runs(a) && moe_tile_fits(a, dtype);
   switch (dtype) {
     case kBF16: launch_ffn<kBF16>(a, fast_gu, fast_dn, small, tile && fast_gu, tile && fast_dn, stream); break;
     case kF16: launch_ffn<kF16>(a, fast_gu, fast_dn, small, tile && fast_gu, tile && fast_dn, stream); break;
