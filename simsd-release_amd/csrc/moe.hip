@@ -841,16 +841,16 @@ namespace {
 
 // Slots an expert holds on average from which the grouped projections take
 // runs of tiles (moe_tile.hip); below, each tile streams its expert's weights
-// by itself, over as many more workgroups.  Experts whose columns fill the chip
-// several times (10 workgroups a CU of gate/up, one run an expert) gain from 11
-// slots on, others from 18.  Single tiles over runs, us a layer, at 10 / 11 /
-// 14 / 18 slots: 256 experts x 512 columns 1.02 1.08 1.22 1.47; 128 x 768 0.99
-// 0.98 1.12 1.43; 8 x 14336 0.96 1.03 1.11 1.47; 16 x 6400 0.98 1.00 1.19 1.33;
-// 64 x 1024 0.88 0.90 0.98 1.21; 16 x 1024 0.85 0.87 0.90 1.11; 8 x 2048 0.77
-// 0.77 0.83 1.07; 8 x 5632 0.92 0.95 1.09 1.21.
-constexpr int64_t kRunMinSlots = 11, kRunMinSlotsFew = 18, kRunColumns = 10 * 256 * 32;
+// by itself, over as many more workgroups.  The more workgroups of gate/up a CU
+// has at one run an expert (10, 4, fewer), the sooner runs gain.  Single tiles
+// over runs, us a layer, at 10 / 11 / 13 / 14 / 16 / 18 slots: 256 experts x 512
+// columns 1.02 1.08 1.07 1.1 1.2 1.3; 16 x 6400 0.98 1.00 - 1.19 1.21 1.33;
+// 64 x 1024 0.94 0.92 1.04 1.08 1.20 1.21, with a shared expert 0.92 1.01 1.07
+// 1.17 1.20 1.30; 32 x 1024 0.87 0.89 1.05 1.07 1.07 1.39; 16 x 1024 0.85 0.87 -
+// 0.90 1.10 1.11; 8 x 2048 0.77 0.77 - 0.83 0.89 1.07.
 bool takes_runs(const MoeArgs& a) {
-  return a.T * a.k >= (a.E * a.I >= kRunColumns ? kRunMinSlots : kRunMinSlotsFew) * a.E;
+  const int64_t columns = (int64_t)a.E * a.I;   // 32 of them a workgroup
+  return a.T * a.k >= (columns >= 10 * 256 * 32 ? 11 : columns >= 4 * 256 * 32 ? 13 : 18) * (int64_t)a.E;
 }
 
 inline int esize_of(int dtype) { return dtype == kF32 ? 4 : 2; }
