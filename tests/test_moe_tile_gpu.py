@@ -2,19 +2,33 @@
 16-slot tile on average) and the wide combine, at the edges of the runs: slot
 counts per expert around 16, 64 and 128, empty experts, one expert with
 everything, invalid ids, ragged H and I, a shared expert with a partial run,
-more slots than one scatter span -- against the oracle on small-integer data,
-where every sum is exact, and bit for bit against the single-tile kernels."""
+more slots than one scatter span -- equal bit for bit to the oracle and to the
+single-tile kernels, on data whose every step is exact: gates are 0 or at least
+32, where silu(g) is 0 or rounds to g, and the sums are of small integers."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
+from oracle import moe as omoe
 
 DEV = "cuda"
 
 
 def _ints(g, *shape, lo=-2, hi=3, dtype=torch.bfloat16):
     return torch.randint(lo, hi, shape, generator=g).to(dtype).to(DEV)
+
+
+def _sparse(g, *shape, values, dtype):
+    """One entry in eight from ``values``, the others zero: the steps' sums then
+    stay below fp16's 65504 (the largest |y| of these sizes is 1.3e4)."""
+    pick = torch.tensor(values)[torch.randint(0, len(values), shape, generator=g)]
+    return (pick * (torch.rand(shape, generator=g) < 0.125)).to(dtype).to(DEV)
+
+
+def _np(t):
+    return t.float().cpu().numpy().astype(np.float64)
 
 
 def _ids(pattern, T, k, E, g):
@@ -38,19 +52,19 @@ def _ids(pattern, T, k, E, g):
 @pytest.mark.parametrize("pattern,T,k,E,H,I,Is", [("edges", 200, 4, 16, 128, 64, 64), ("one", 130, 3, 8, 72, 40, 0),
                                                   ("spread", 64, 2, 4, 264, 96, 32), ("spread", 333, 8, 64, 136, 72, 40),
                                                   ("invalid", 150, 4, 8, 64, 24, 24), ("spread", 1000, 8, 16, 64, 32, 0),
-                                                  ("spread", 77, 1, 3, 128, 33 * 8, 8)])
-def test_runs_equal_single_tiles(pattern, T, k, E, H, I, Is, dtype):
+                                                  ("spread", 77, 1, 3, 128, 33 * 8, 8), ("spread", 96, 8, 64, 64, 1280, 0)])
+def test_runs_equal_oracle_and_single_tiles(pattern, T, k, E, H, I, Is, dtype):
     from kernels.moe_dispatch_fused import _align, _grouped_ffn, _num_tiles
     print(f"moe runs {pattern} T={T} k={k} E={E} H={H} I={I} Is={Is} {dtype}", flush=True)
     g = torch.Generator().manual_seed(T + E)
     ids = _ids(pattern, T, k, E, g)
-    assert T * k >= 10 * E                 # the rule's side with runs
-    x = _ints(g, T, H, lo=-1, hi=2, dtype=dtype)
-    wg, wu, wd = (_ints(g, E, I, H, lo=-1, hi=2, dtype=dtype), _ints(g, E, I, H, lo=-1, hi=2, dtype=dtype),
-                  _ints(g, E, H, I, lo=-1, hi=2, dtype=dtype))
-    tw = torch.rand(T, k, generator=g).to(DEV)
-    shared = ((_ints(g, Is, H, lo=-1, hi=2, dtype=dtype), _ints(g, Is, H, lo=-1, hi=2, dtype=dtype),
-               _ints(g, H, Is, lo=-1, hi=2, dtype=dtype)) if Is else None)
+    assert T * k >= (11 if E * I >= 10 * 256 * 32 else 18) * E     # the rule's side with runs
+    x = _sparse(g, T, H, values=[1.0], dtype=dtype)
+    wg, wu, wd = (_sparse(g, E, I, H, values=[32.0], dtype=dtype), _ints(g, E, I, H, lo=-1, hi=2, dtype=dtype),
+                  _sparse(g, E, H, I, values=[-1.0, 1.0], dtype=dtype))
+    tw = (torch.randint(1, 257, (T, k), generator=g) / 256).to(DEV)   # products with the y (multiples of 32) exact
+    shared = ((_sparse(g, Is, H, values=[32.0], dtype=dtype), _ints(g, Is, H, lo=-1, hi=2, dtype=dtype),
+               _sparse(g, H, Is, values=[-1.0, 1.0], dtype=dtype)) if Is else None)
     slots, te = _align(ids, E, _num_tiles(T * k, E))
     with torch.inference_mode():
         got = _grouped_ffn(x, ids, tw, wg, wu, wd, slots, te, shared=shared)
@@ -63,13 +77,13 @@ def test_runs_equal_single_tiles(pattern, T, k, E, H, I, Is, dtype):
         one = _grouped_ffn(x, ids1, tw, *big, slots, te1, shared=shared)
         wide = torch.zeros(T, 2 * H, dtype=dtype, device=DEV)    # outputs 2 apart: the narrow combine
         _grouped_ffn(x, ids, tw, wg, wu, wd, slots, te, shared=shared, out=wide[:, ::2])
-    # integer products: the gate and up sums are exact on both sides, so h is
-    # equal; the down sums of 16-bit h differ at most by their fp32 order
-    ref = one.float()
-    tol = 2.0 ** -7 * float(ref.abs().max()) + 1e-3
-    assert float((got.float() - ref).abs().max()) <= tol
-    assert float((wide[:, ::2].float() - got.float()).abs().max()) == 0.0 and not wide[:, 1::2].any()
-    assert torch.isfinite(got).all()
+    ref = omoe.dispatch_grouped(_np(x), ids.cpu().numpy(), _np(tw), _np(wg), _np(wu), _np(wd),
+                                dtype={torch.bfloat16: "bf16", torch.float16: "fp16"}[dtype],
+                                shared=None if shared is None else tuple(_np(w) for w in shared))
+    assert np.abs(ref).max() > 32 and np.isfinite(ref).all()
+    assert np.array_equal(_np(got), ref)
+    assert torch.equal(one, got)
+    assert torch.equal(wide[:, ::2], got) and not wide[:, 1::2].any()
 
 
 @pytest.mark.gpu

@@ -44,6 +44,29 @@ def test_reduce_of_partials_wide_equals_narrow(M, dtype):
 
 @pytest.mark.gpu
 @DTYPES
+@pytest.mark.parametrize("M", [1, 17, 261])
+def test_gated_reduce_wide_equals_narrow(M, dtype):
+    """The same of the gated sum (gate and up partials, SiLU.mul): contiguous
+    outputs against odd rows at an address that is not 8-byte aligned."""
+    from kernels import _native
+    g = torch.Generator(device=DEV).manual_seed(M)
+    lib, code = _native.lib(), _native.DTYPE_CODES[dtype]
+    for K, I, split in [(1024, 4, 2), (1000, 260, 3), (1024, 4100, 4)]:
+        print(f"gated reduce M={M} K={K} I={I} split={split} {dtype}", flush=True)
+        x = torch.randn(M, K, device=DEV, generator=g).to(dtype)
+        w = (torch.randn(2 * I, K, device=DEV, generator=g) * K ** -0.5).to(dtype)
+        outs = torch.zeros(M, I, dtype=dtype, device=DEV), _off_by_one(torch.zeros(M, I, dtype=dtype, device=DEV))
+        ws = torch.empty(split * M * 2 * I * 4, dtype=torch.uint8, device=DEV)
+        for h in outs:
+            st = lib.simsd_thin_linear_silu_mul(x.data_ptr(), K, 1, w[:I].data_ptr(), K, 1, w[I:].data_ptr(), K, 1,
+                                                h.data_ptr(), h.stride(0), 1, M, I, K, code, 16, 0, split, 4,
+                                                ws.data_ptr(), ws.numel(), _native.stream_of(h.device))
+            _native.check(st, "thin_linear_silu_mul")
+        assert torch.equal(*outs) and outs[0].abs().max() > 0, (K, I)
+
+
+@pytest.mark.gpu
+@DTYPES
 @pytest.mark.parametrize("M", [683, 1024, 1025])
 def test_rope_cache_rows_equal_single_tokens(M, dtype):
     """One call over M tokens equals M / 64 calls of few: slots in aligned

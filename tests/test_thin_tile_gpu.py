@@ -5,6 +5,8 @@ it hands back to the row-block kernels.  Integer data, so every sum is exact
 and the outputs equal the oracle's bit for bit."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -61,13 +63,23 @@ def test_tile_edges_bit_exact(M, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("M,N,K,gated", [
-    (700, 4096, 520, False), (385, 3001, 1000, True),                                  # 128 x 128
-    (1025, 6141, 72, False), (260, 2048, 12288, False), (1025, 4099, 520, True),       # 256 x 128; a split of 8
-    (640, 12300, 256, False), (300, 8195, 8192, False), (513, 6200, 2048, True)])      # 128 x 256; a split of 2
-def test_prompt_tiles_vs_oracle(M, N, K, gated, dtype):
-    """The 8-wave tiles at sizes that choose them, partial last tiles and
-    stages: integer data bit for bit, gated within the oracle's bound."""
+@pytest.mark.parametrize("M,N,K,gated,plan", [       # plan: weight rows and tokens of the tile, split
+    (260, 6140, 2048, False, (128, 64, 1)), (257, 3070, 4096, True, (128, 64, 1)),
+    (700, 4096, 520, False, (128, 128, 1)), (385, 3001, 1000, True, (128, 128, 1)), (260, 2048, 12288, False, (128, 128, 4)),
+    (133, 3071, 4096, True, (128, 128, 2)), (257, 12288, 4096, True, (128, 128, 1)), (700, 1028, 8192, True, (128, 128, 2)),
+    (640, 12300, 256, False, (256, 128, 1)), (513, 6200, 2048, True, (256, 128, 1)), (300, 4100, 12288, False, (256, 128, 4)),
+    (513, 1499, 12288, True, (256, 128, 4)),
+    (1025, 6141, 72, False, (128, 256, 1)), (1025, 4099, 520, True, (128, 256, 1)), (1024, 4096, 12288, False, (128, 256, 2)),
+    (300, 1499, 12288, True, (128, 256, 4)), (700, 1500, 12288, True, (128, 256, 2))])
+def test_prompt_tiles_vs_oracle(M, N, K, gated, plan, dtype):
+    """The tiles above 64 tokens at sizes that choose them, plain and gated,
+    with and without partials (summed four outputs a thread or, for odd N, one),
+    partial last tiles and stages: integer data bit for bit, gated within the
+    oracle's bound."""
+    from kernels import _native
+    out = (ctypes.c_int * 4)()
+    assert _native.lib().simsd_thin_linear_plan(M, 2 * N if gated else N, K, _native.DTYPE_CODES[dtype], -1, 0, 4, out) == 0
+    assert (out[0], out[1], out[3]) == plan, "the plan takes another tile here: choose a size that takes this one"
     from kernels.thin_linear_fused import thin_linear_residual, thin_linear_silu_mul
     print(f"prompt tiles M={M} N={N} K={K} gated={gated} {dtype}", flush=True)
     with torch.inference_mode():
