@@ -233,7 +233,7 @@ def cpu_baseline_linear(torch, workload, M):
 
 
 def run_linear(args, torch, dev):
-    from kernels.thin_linear_fused import thin_linear
+    from kernels.thin_linear_fused import TILE, pick_config, thin_linear
 
     M, calls = make_linear_calls(torch, dev, args.workload)
     step_bytes = sum(linear_bytes(M, x.shape[1], w.shape[0]) for _, x, w in calls)
@@ -293,9 +293,14 @@ def run_linear(args, torch, dev):
 
     gbs = step_bytes / (ms * 1e-3) / 1e9
     avg_launch_us = ms * 1e3 / launches
-    kernel = ("thin_gemv4_kernel (4x4x4 MFMA GEMV, M <= 8)" if M <= 8 else
-              "thin_gemm_lds_kernel (16x16x32 MFMA via LDS; per call, the split-K reduce "
-              "launch of down_proj included)")
+    if M <= 8:
+        kernel = "thin_gemv4_kernel (4x4x4 MFMA GEMV, M <= 8)"
+    else:
+        tiled = [n for n, d in per_op.items() if pick_config(M, d["N"], d["K"])[1] == TILE]
+        rows = [n for n in per_op if n not in tiled]
+        kernel = " and ".join(f"{k} ({', '.join(ops)})" for k, ops in (
+            ("thin_tile_kernel", tiled), ("thin_gemm_lds_kernel / thin_gemm_xs_kernel", rows)) if ops)
+        kernel += "; per call, the launch that sums a split's partials included"
     breakdown = {
         n: {"K": d["K"], "N": d["N"], "calls": d["calls"], "us_per_call": round(d["us"], 3),
             "GB/s": round(d["bytes"] / (d["us"] * 1e-6) / 1e9, 1),

@@ -941,7 +941,7 @@ SIMSD_DEV u32x4_t norm_rope16(u32x4_t x, u32x4_t w, bool has_w, u32x4_t c, u32x4
 // are no aligned run), 512 tokens 11.3 -> 6.5, 200 tokens 6.0 -> 4.4.
 // The same sums and rounding points: the outputs are the same bits.
 constexpr int kRopeToks = 4;
-constexpr int64_t kRopeRowsMin = 4096;
+constexpr int64_t kRopeRowsMin = 8192;
 
 template <int DT>
 SIMSD_DEV void put_v16(char* base, int64_t s, bool ok, bool run, int j, int tk, u32x4_t v) {
@@ -1596,10 +1596,11 @@ extern "C" int simsd_qkv_rope_cache(const void* qkv, int64_t sqkv, const void* q
   const int waves = heads < 8 ? heads : 8;
   const dim3 grid((unsigned)M, (unsigned)((heads + waves - 1) / waves));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // Four tokens a wave where one a wave is more than half of the chip's 8192
-  // waves (133 tokens x 48 heads: 4.0 us, or 4.75 off an aligned run, against
-  // 4.8); below it the 2-byte V stores of a run off its alignment cost more
-  // than the wider rows give (100 tokens x 32 heads: 3.7 or 4.5 against 4.0).
+  // Four tokens a wave where one a wave is more than the chip's 8192 waves.
+  // The slots are on the device: where the tokens' are no aligned run, V goes
+  // out in 2-byte stores, and the wider rows gain only from there on.  One token
+  // / four, us, 48 heads, 94 tokens: 4.66 / 4.31 aligned, 4.71 / 5.01 off by one,
+  // 4.65 / 5.08 in any order; 175 tokens 6.12 / 4.89, 6.12 / 5.55, 6.01 / 5.85.
   // Its 16-byte rows leave other strides and addresses to the one-token form.
   const bool rows16 = al(qkv, 16) && sqkv % 8 == 0 && al(cos, 16) && al(sin, 16) && scs % 8 == 0 &&
                       al(q_norm_w, 16) && al(k_norm_w, 16) && al(k_cache, 16) && al(v_cache, 8) &&
