@@ -7,9 +7,9 @@
 // consecutive tiles of one expert as one 64-row activation tile of the linear
 // layers' tile kernel, whose activation loads gather the slots' rows (every
 // load into LDS has its own address), and the weights are read once for it.
-// 1001 tokens, H 2048, I 512: gate_up 266 us (4.0 TB/s of weights), down 161;
-// the step, with the align kernel's parallel scatter and the wide combine,
-// 899 -> 433.  What bounds it now is streaming 32 (gate_up) and 8 (down)
+// 1001 tokens, H 2048, I 512 (traced): gate_up 258 us (4.2 TB/s of weights),
+// down 155; the case's step, with the align kernel's parallel scatter and the
+// wide combine, 893 -> 447.  What bounds it now is streaming 32 (gate_up) and 8 (down)
 // stages per short-lived workgroup, and the workgroups of the tiles that are
 // not the first of a run, which exit after a load.
 #include "moe_common.hpp"

@@ -1177,7 +1177,9 @@ void launch_xs(const ThinPlan& pl, const ThinArgs& args, hipStream_t stream) {
 }
 
 // (rb, ks) of a shared-activation plan: (2, 2), (2, 3), (2, 4); ungated also
-// (1, 4), (1, 8)
+// (1, 4), (1, 8).  Automatic calls take these at 9 to 16 tokens, ungated; the
+// gated and the wider forms serve explicit block_n 64 to 128 (above 16 tokens
+// the tile kernel is the faster on all operands they take).
 template <int DT, int CB, bool GLU>
 void xs_shape(const ThinPlan& pl, const ThinArgs& args, hipStream_t stream) {
   if (pl.rb == 2) {

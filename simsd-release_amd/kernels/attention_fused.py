@@ -20,9 +20,10 @@ several, the last of which merges their partials; two launches past it
 (chunked partials, then their merge).  More rows take chunked partials through
 LDS (csrc/attn_tile.hip), merged by a second launch unless one chunk covers
 the keys, or, up to 128 rows over short contexts, 64-key chunks without LDS.
-The form and the chunking follow the host's ``valid_len`` bound, so a caller replaying graphs over a growing
-context captures one graph per bound; ``valid_len_dev`` then lowers the
-length at run time, and the kernels trim their work to it.  The cache
+The form and the chunking follow the host's ``valid_len`` bound, so a caller
+replaying graphs over a growing context captures one graph per bound;
+``valid_len_dev`` then lowers the length at run time, and the kernels trim
+their work to it.  The cache
 (``BlockKVCache``) keeps one copy of each KV head (no per-query-head replicas)
 in tiles laid out in the order the attention kernels read them, so every
 wave-wide load covers 1 KB of contiguous memory; ``keys`` / ``values`` /

@@ -61,8 +61,9 @@ column-block width (heuristic: 4 or 8 for the GEMV, 16, 32 or 48 otherwise),
 BLOCK_N the weight rows per workgroup (4, 8, 16, 24, 32, 64, 96 or 128; other
 values round down to one of these; at least 16 above 8 tokens; 64, 96 and 128
 apply above 8 tokens in bf16/fp16 and act as 32 elsewhere; 24 applies to the
-ungated projection above 8 tokens and acts as 16 elsewhere), BLOCK_K the K elements of
-activations a wave holds at once in the GEMV (256 or 1024), SPLIT_K the workgroups along K, num_warps the waves per workgroup (2, 4 or 8);
+ungated projection above 8 tokens and acts as 16 elsewhere), BLOCK_K the K
+elements of activations a wave holds at once in the GEMV (256 or 1024), SPLIT_K
+the workgroups along K, num_warps the waves per workgroup (2, 4 or 8);
 num_stages is accepted and ignored.  BLOCK_N -1 (``TILE``) is the tile kernel,
 which picks its tile by the sizes, and with SPLIT_K 0 its split; BLOCK_K and
 num_warps mean nothing to it.
@@ -137,7 +138,10 @@ def reset_workspace() -> None:
 # workgroup x waves x split on one MI355X (M=4 for draft shapes, M=16 and 32
 # for target shapes; bf16; HIP graph over a >= 1 GiB weight pool so the
 # 256 MB MALL cannot serve repeats).  Entries not swept directly (separate
-# gate/up, k/v and lm_head of the target) follow the nearest swept shape.
+# gate/up, k/v and lm_head of the target) follow the nearest swept shape.  The
+# times are the row-block kernels' own; above 16 tokens most of these shapes
+# take the tile kernel (_takes_tile), and the entries serve the shapes it
+# leaves, explicit num_warps and operands it does not take.
 TUNED: dict[tuple[int, int], tuple[int, int, int, int, int, int]] = {
     # SDAR-1.7B draft projections (hidden 2048, 16 q / 8 kv heads, inter 6144)
     (2048, 2048): (16, 8, 1024, 1, 2, 2),     # q_proj, o_proj      4.0 us
